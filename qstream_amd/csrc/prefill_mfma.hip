@@ -661,7 +661,7 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 4) void prefill_few_kernel(FewArgs 
     const size_t row_bytes = (size_t)a.nb * BB;
 
     // Chunk c into buffer `buf`: wave w loads rows 2 w and 2 w + 1 (rows past
-    // n and units past the row repeat the last one; such units meet zeros of x)
+    // n and units past the row repeat the last one; neither is used)
     auto load_chunk = [&](int c, uint8_t* buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int h = 0; h < 2 * NT; h++) {
@@ -748,8 +748,10 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 4) void prefill_few_kernel(FewArgs 
             const uint8_t* buf = few_lds + i * NT * FEW_CHUNK;
 #pragma unroll
             for (int v = 0; v < 8; v++) {
-                if ((c0 + i) * FEW_U + 8 * v >= nu) break;
                 const int ul = 8 * v + wave;              // unit of the chunk
+                // (no unit of columns past k, where x is zero: an infinite scale
+                // or zero times that is NaN)
+                if (64 * ((c0 + i) * FEW_U + ul) >= a.k) break;
                 const uint32_t slot = (uint32_t)(n16 * 1024 + ((ul ^ n16) << 4));
                 const uint32_t ts = (uint32_t)(FEW_T + n16 * 256 + (((ul + 4 * n16) & 63) << 2));
                 uint32_t o0, o1, om;

@@ -77,6 +77,25 @@ def test_special_values(hip, m, bs):
     assert np.array_equal(got[np.ix_(keep_t, keep_r)].view(np.uint32), clean[np.ix_(keep_t, keep_r)].view(np.uint32))
 
 
+@pytest.mark.parametrize("off,m", [(0, 2), (2, 2), (0, 40), (2, 40)])
+@pytest.mark.parametrize("k,bs", [(64, 64), (576, 64), (4160, 64), (136, 128), (264, 256), (512, 256)])
+def test_infinite_last_block(hip, k, bs, off, m):
+    """A last block whose scale or zero is Inf gives Inf, as the scalar matvec
+    does for x > 0 and codes > 0, whatever the row's unit count leaves of a
+    round of the waves (units past the row add nothing, not Inf * 0)."""
+    n = 20
+    payload, _ = case(k, m, n, k, bs)
+    xb = np.full((m, k), 0x3F80, np.uint16)                     # 1.0
+    p = np.frombuffer(payload, np.uint8).copy()
+    nb, bb = (k + bs - 1) // bs, 4 + bs // 2
+    blocks = p[:n * nb * bb].reshape(n, nb, bb)
+    blocks[5, nb - 1, 4:] |= 0x11                               # codes of at least 1
+    blocks[5, nb - 1, off:off + 2] = np.frombuffer(np.uint16(0x7C00).tobytes(), np.uint8)
+    got = run(hip, p, xb, m, n, k, bs)
+    assert np.isposinf(got[:, 5]).all()
+    assert np.isfinite(np.delete(got, 5, axis=1)).all()
+
+
 # shapes whose tiles of 112 need a second round of 256 workgroups and whose
 # tiles of 128 do not: full and partial last tiles both ways, every block
 # size, ragged k, rows of more blocks than the wide tile's zero stash holds
