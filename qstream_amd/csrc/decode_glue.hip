@@ -350,8 +350,7 @@ __global__ __launch_bounds__(64) void rope_kv_kernel(float* q, float* k, const f
 //
 // Bound by the cache bytes (2 (hd + 4) a position and KV head) and, short of
 // a few thousand positions, by its chain of one load and three barriers.
-// Every
-// byte of the chunk (and its scales) is requested before any is used, as
+// Every byte of the chunk (and its scales) is requested before any is used, as
 // 16-byte pieces; thread t holds pieces t, t + 256, ..., i.e. dims
 // 16 (t % HC) .. + 15 of positions (t + 256 j) / HC, for K and V alike, so a
 // wave's load covers 1 KB of consecutive rows.
@@ -591,10 +590,31 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_chunk_kernel(AttArgs a)
     if (wave < G) {
         const float inv_sqrt_d = __fdiv_rn(1.0f, __fsqrt_rn((float)HD));
         float sc[2];
+        bool wide = false;
 #pragma unroll
-        for (int e = 0; e < 2; e++)
-            sc[e] = lane + 64 * e < np ? qsf::mul_rn(qsf::mul_rn(dots[wave][lane + 64 * e], kscale[e]), inv_sqrt_d)
-                                       : -INFINITY;
+        for (int e = 0; e < 2; e++) {
+            sc[e] = qsf::mul_rn(dots[wave][lane + 64 * e], kscale[e]);
+            wide |= !(__builtin_fabsf(sc[e]) < INFINITY);
+        }
+        // The codes' sum can pass fp32's range (q from 2^113 on) where the
+        // dequantised row's does not, and an Inf scale times a zero code is
+        // NaN: such positions take their rows element by element.
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(wide) != 0, 0)) {
+#pragma unroll 1
+            for (int e = 0; e < 2; e++) {
+                const int p = lane + 64 * e;
+                const float scale = e ? kscale[1] : kscale[0], d = e ? sc[1] : sc[0];
+                if (p >= np || __builtin_fabsf(d) < INFINITY) continue;
+                const int8_t* row = last && p == np - 1 ? newc[0] : a.kc + (row0 + p) * HD;
+                float x = 0.f;
+#pragma unroll 1
+                for (int c = 0; c < HD; c++) x = fmaf(qs[wave * HD + c], qsf::mul_rn((float)row[c], scale), x);
+                if (e) sc[1] = x;
+                else sc[0] = x;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 2; e++) sc[e] = lane + 64 * e < np ? qsf::mul_rn(sc[e], inv_sqrt_d) : -INFINITY;
         const float m = wave_max64(fmaxf(sc[0], sc[1]));
         float l = 0.f;
 #pragma unroll

@@ -71,3 +71,52 @@ def test_grouped_heads(hip, oracle, nh, nkv, hd, position):
     rope.free()
     for name, x, y in zip(("kc", "vc", "ks", "vs", "out"), *outs):
         assert np.array_equal(x, y), name
+
+
+@pytest.mark.parametrize("nh,nkv,hd,position", [(8, 2, 128, 300), (4, 4, 64, 127), (8, 1, 256, 4223), (32, 8, 128, 4100)])
+def test_large_queries_and_infinite_scales(hip, oracle, nh, nkv, hd, position):
+    """Queries whose products with the codes alone pass fp32's range while those
+    with the dequantised row do not (plain call, and the fused one, whose new
+    row of 1e-29 takes most heads' weight or none of it), and an Inf scale over a row with a zero code: NaN for the
+    heads of that KV head, the others untouched."""
+    torch = torch_cuda()
+    rng = np.random.default_rng(hd + position)
+    max_seq, g = position + 1, nh // nkv
+    kc = rng.integers(-127, 128, (nkv, max_seq, hd)).astype(np.int8)
+    vc = rng.integers(-127, 128, (nkv, max_seq, hd)).astype(np.int8)
+    tiny = np.float32(2.0) ** np.float32(-120)
+    ks = (rng.random((nkv, max_seq)) * 0.02).astype(np.float32) * tiny
+    vs = (rng.random((nkv, max_seq)) * 0.02).astype(np.float32)
+    q = rng.standard_normal(nh * hd).astype(np.float32) / tiny
+    out = torch.full((nh * hd,), np.nan, device="cuda:0")
+    hip.attention(dev(q), dev(kc), dev(vc), dev(ks), dev(vs), max_seq, nh, nkv, hd, position, out, stream=_s())
+    got = host(out)
+    assert np.isfinite(got).all()
+    assert rel_l2(got, oracle.attention(q, kc, vc, ks, vs, max_seq, nh, nkv, hd, position)) <= REL_L2
+
+    rope = hip.Rope(hd, 10000.0)
+    k, v = (rng.standard_normal(nkv * hd).astype(np.float32) * np.float32(0.3) for _ in range(2))
+    dq, dk, dv = dev(q), dev(k * np.float32(1e-29)), dev(v)
+    a = [dev(x.copy()) for x in (kc, vc, ks, vs)]
+    outs = []
+    for fused in (False, True):
+        b, o = [x.clone() for x in a], torch.full((nh * hd,), np.nan, device="cuda:0")
+        q2, k2 = dq.clone(), dk.clone()
+        if fused:
+            rope.apply_store_attend(q2, k2, dv, nh, nkv, position, *b, max_seq, o, stream=_s())
+        else:
+            rope.apply_and_store(q2, k2, dv, nh, nkv, position, *b, max_seq, stream=_s())
+            hip.attention(q2, *b, max_seq, nh, nkv, hd, position, o, stream=_s())
+        outs.append(host(o))
+    rope.free()
+    assert np.isfinite(outs[0]).all() and np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+    q, ks, p = q * tiny, ks / tiny, position // 2
+    clean = torch.full((nh * hd,), np.nan, device="cuda:0")
+    hip.attention(dev(q), dev(kc), dev(vc), dev(ks), dev(vs), max_seq, nh, nkv, hd, position, clean, stream=_s())
+    kc[0, p, 3], ks[0, p] = 0, np.inf
+    hip.attention(dev(q), dev(kc), dev(vc), dev(ks), dev(vs), max_seq, nh, nkv, hd, position, out, stream=_s())
+    got = host(out)
+    assert np.isnan(oracle.attention(q, kc, vc, ks, vs, max_seq, nh, nkv, hd, position)[:g * hd]).all()
+    assert np.isnan(got[:g * hd]).all()
+    assert np.array_equal(got[g * hd:].view(np.uint32), host(clean)[g * hd:].view(np.uint32))
