@@ -34,7 +34,7 @@ typedef struct qsf_hip_tensor {
     const void* host_key;       /* registry key (host payload pointer) */
     size_t   payload_bytes;     /* on-disk payload size (algorithmic bytes) */
     uint8_t* d_blocks;          /* rows*nb*block_bytes (MXFP4: codes plane) */
-    uint8_t* d_scales;          /* MXFP4: E8M0 plane, rows of qk_mx_ld(nb), else NULL */
+    uint8_t* d_scales;          /* MXFP4: E8M0 plane, else NULL */
     uint32_t n_outliers;        /* entries in the file table */
     uint32_t n_csr;             /* entries kept (in range) */
     uint32_t* d_row_ptr;        /* rows+1, or NULL */
@@ -47,8 +47,6 @@ typedef struct qsf_hip_tensor {
     int      frag_nq;           /* fragment order: 4-block quads a row, ceil(nb / 4) */
     int      plane;             /* 1: d_blocks in row-plane order (below); with frag
                                  * 0 as well: on-disk order */
-    int      mx_wide;           /* MXFP4: a block scale is 2^126 or 2^127 (codes 4 and 6 times
-                                 * it are outside bf16) */
     int      registry_owned;    /* uploaded implicitly by a table-slot call */
     const void* succ;           /* table slots: the key called next with the same x ... */
     int      succ_hits;         /* ... this many times since it last differed */
@@ -58,14 +56,20 @@ typedef struct qsf_hip_tensor {
 
 #define QK_MAX_GROUP 8
 
-/* Blocks from row to row of an MXFP4 tensor's device planes (nb used, the
- * rest zero): whole 128-byte lines of codes. */
+/* MXFP4 device order, of the codes (16 bytes a block) and of the scales (1
+ * byte) alike: the whole groups of 8 blocks of every row, row after row, then
+ * the nb % 8 blocks left of every row, row after row.  As many bytes as on
+ * disk, and a group's codes are a 128-byte line of their own.  Place of block
+ * b of a row: */
 #ifdef __cplusplus
-constexpr
-#else
-static inline
+__host__ __device__ inline size_t qk_mx_at(int rows, int nb, int row, int b) {
+    const int whole = nb & ~7;
+    return b < whole ? (size_t)row * whole + b : (size_t)rows * whole + (size_t)row * (nb - whole) + (b - whole);
+}
 #endif
-int qk_mx_ld(int nb) { return (nb + 7) & ~7; }
+/* Bytes of the scales' allocation past their end: the last row's remainder
+ * is read as 8 bytes. */
+#define QK_MX_SLACK 8
 
 /* Fragment order: the device layout of a dense tensor the matrix-core GEMV
  * covers (qk_mfma_layout).  The on-disk blocks, unchanged, regrouped into
@@ -199,6 +203,13 @@ size_t qk_moe_ws_bytes(int n_exp, int k, int ntok, int hidden, int eid);
 int qk_moe_launch(const qk_mx_expert* d_experts, int n_exp, int k, int norm, int act,
                   int hidden, int eid, int ntok, const float* d_x, const float* d_logits,
                   float* d_out, void* d_ws, int stages, hipStream_t s);
+
+/* Rows r0 .. r0 + n - 1 of an MXFP4 tensor, from on-disk order (codes, scales)
+ * to the tensor's planes. */
+int qk_mx_split(const uint8_t* codes, const uint8_t* scales, uint8_t* d_blocks, uint8_t* d_scales, size_t rows,
+                size_t r0, size_t n, int nb, hipStream_t s);
+/* *d_flag = whether a block scale of the experts is 2^126 or 2^127. */
+int qk_mx_wide(const qk_mx_expert* d_experts, int n_exp, int hidden, int eid, int* d_flag, hipStream_t s);
 
 /* The FFN for more than 8 tokens in one pass on the matrix cores: up to
  * qk_moe_many_tokens(k) tokens, with a workspace of qk_moe_many_ws_bytes. */

@@ -62,7 +62,7 @@ typedef struct {
     hipStream_t stream;
     void* ws;          size_t ws_bytes;       /* prefill workspace */
     void* att_ws;      size_t att_ws_bytes;   /* attention partials */
-    void* h_up;        size_t h_up_bytes;     /* pinned: an upload's padded rows */
+    void* d_up;        size_t d_up_bytes;     /* a piece of an MXFP4 upload, in on-disk order */
     float* d_x;        size_t d_x_n;          /* device copy of a table slot's x */
     void* slot_xq;     size_t slot_xq_bytes;  /* a table slot's prepared x */
     int xq_ok, xq_fmt, xq_bs, xq_cols;        /* slot_xq and d_x hold h_x prepared so */
@@ -404,41 +404,33 @@ static void plane_permute(uint8_t* dst, const uint8_t* src, int rows, int nb, in
     }
 }
 
-/* An MXFP4 payload to the tensor's planes, rows padded with zeros (qk_mx_ld):
- * the rows are laid out in two halves of a pinned buffer by turns, so one
- * half's transfer runs while the other is filled.  (With a copy on the device
- * that a kernel padded, uploads of 96 tensors of 2880 x 2880 between other
- * work took 152 ms against 81 unpadded; this way no longer than unpadded.)
- * Done when it returns: a caller may use the tensor on any stream. */
-#define UP_HALF ((size_t)4 << 20)
-static hipError_t mx_copy(qsf_hip_tensor* t, const uint8_t* payload, size_t bytes) {
-    if (bytes == 0) return hipSuccess;
-    const size_t rows = (size_t)t->rows, nb = (size_t)t->nb, ld = (size_t)qk_mx_ld(t->nb);
+/* An MXFP4 payload to the tensor's planes (qk_mx_at).  Where that is the
+ * on-disk order (a multiple of 8 blocks a row, or fewer than 8) as it is;
+ * else by the piece through a device buffer, from which a kernel moves each
+ * row's whole groups of 8 blocks and its remainder to their planes.  Done when it
+ * returns: a caller may use the tensor on any stream. */
+#define UP_PIECE ((size_t)8 << 20)
+static hipError_t mx_copy(qsf_hip_tensor* t, const uint8_t* payload) {
+    const size_t rows = (size_t)t->rows, nb = (size_t)t->nb;
     const uint8_t* scales = payload + rows * nb * 16;
-    if (nb == ld) {
+    if (rows * nb == 0) return hipSuccess;
+    if (nb % 8 == 0 || nb < 8) {
         const hipError_t he = hipMemcpy(t->d_blocks, payload, rows * nb * 16, hipMemcpyHostToDevice);
         return he != hipSuccess ? he : hipMemcpy(t->d_scales, scales, rows * nb, hipMemcpyHostToDevice);
     }
-    const size_t step = UP_HALF / (ld * 17) ? UP_HALF / (ld * 17) : 1;      /* rows a half */
-    const size_t half = step * ld * 17 > UP_HALF ? step * ld * 17 : UP_HALF;
-    if (ensure_host(&g_dev.h_up, &g_dev.h_up_bytes, 2 * half) != E_OK) return hipErrorOutOfMemory;
+    const size_t step = UP_PIECE / (nb * 17) ? UP_PIECE / (nb * 17) : 1;    /* rows a piece */
+    if (ensure_dev(&g_dev.d_up, &g_dev.d_up_bytes, nb * 17 > UP_PIECE ? nb * 17 : UP_PIECE) != E_OK)
+        return hipErrorOutOfMemory;
+    uint8_t *c = g_dev.d_up, *e = c + step * nb * 16;
     hipError_t he = hipSuccess;
-    int which = 0;
-    for (size_t r = 0; r < rows && he == hipSuccess; r += step, which ^= 1) {
+    for (size_t r = 0; r < rows && he == hipSuccess; r += step) {
         const size_t n = rows - r < step ? rows - r : step;
-        uint8_t *c = (uint8_t*)g_dev.h_up + (which ? half : 0), *e = c + n * ld * 16;
-        if (r && !which && (he = hipStreamSynchronize(g_dev.stream)) != hipSuccess) break;   /* both halves free */
-        for (size_t i = 0; i < n; i++) {
-            memcpy(c + i * ld * 16, payload + (r + i) * nb * 16, nb * 16);
-            memset(c + (i * ld + nb) * 16, 0, (ld - nb) * 16);
-            memcpy(e + i * ld, scales + (r + i) * nb, nb);
-            memset(e + i * ld + nb, 0, ld - nb);
-        }
-        he = hipMemcpyAsync(t->d_blocks + r * ld * 16, c, n * ld * 16, hipMemcpyHostToDevice, g_dev.stream);
-        if (he == hipSuccess)
-            he = hipMemcpyAsync(t->d_scales + r * ld, e, n * ld, hipMemcpyHostToDevice, g_dev.stream);
+        he = hipMemcpyAsync(c, payload + r * nb * 16, n * nb * 16, hipMemcpyHostToDevice, g_dev.stream);
+        if (he == hipSuccess) he = hipMemcpyAsync(e, scales + r * nb, n * nb, hipMemcpyHostToDevice, g_dev.stream);
+        if (he == hipSuccess && qk_mx_split(c, e, t->d_blocks, t->d_scales, rows, r, n, t->nb, g_dev.stream))
+            he = hipErrorLaunchFailure;
     }
-    const hipError_t end = hipStreamSynchronize(g_dev.stream);              /* on an error too: the halves are reused */
+    const hipError_t end = hipStreamSynchronize(g_dev.stream);
     return he != hipSuccess ? he : end;
 }
 
@@ -466,8 +458,6 @@ static qsf_hip_tensor* upload_locked(const void* host, int qt, int rows, int col
         blocks_bytes = (size_t)rows * t->nb * 16;
         scales_bytes = (size_t)rows * t->nb;
         t->payload_bytes = blocks_bytes + scales_bytes;
-        t->mx_wide = scales_bytes && (memchr(p + blocks_bytes, 253, scales_bytes) != NULL ||
-                                      memchr(p + blocks_bytes, 254, scales_bytes) != NULL);
     } else {
         t->nb = (cols + bs - 1) / bs;
         t->block_bytes = 4 + (bs * fmt_bits(fmt) + 7) / 8;
@@ -488,10 +478,7 @@ static qsf_hip_tensor* upload_locked(const void* host, int qt, int rows, int col
               qk_mfma_layout(fmt, bs, cols, is_outlier(qt));
     t->frag_nq = (t->nb + 3) / 4;
     t->plane = !t->frag && rows > 0 && qk_plane_layout(fmt, t->bs);
-    const size_t mx_blocks = fmt < 0 ? (size_t)rows * (size_t)qk_mx_ld(t->nb) : 0;    /* padded */
-    const size_t dev_blocks_bytes = fmt < 0     ? mx_blocks * 16
-                                    : t->frag ? qk_frag_bytes(rows, t->nb, t->block_bytes)
-                                              : blocks_bytes;
+    const size_t dev_blocks_bytes = t->frag ? qk_frag_bytes(rows, t->nb, t->block_bytes) : blocks_bytes;
 
     /* CSR of the outlier table: stable counting sort by row keeps file order
      * within a row; entries with row >= rows are dropped (src/quant.c:432-434). */
@@ -545,7 +532,7 @@ static qsf_hip_tensor* upload_locked(const void* host, int qt, int rows, int col
     /* one allocation: [blocks][scales][row_ptr][ocol][oval], 256-B aligned parts */
     size_t off_blocks = 0;
     size_t off_scales = align256(dev_blocks_bytes);
-    size_t off_rp = off_scales + align256(mx_blocks);
+    size_t off_rp = off_scales + (scales_bytes ? align256(scales_bytes + QK_MX_SLACK) : 0);
     size_t rp_bytes = row_ptr ? ((size_t)rows + 1) * 4 : 0;
     size_t off_oc = off_rp + align256(rp_bytes);
     size_t off_ov = off_oc + align256((size_t)kept * 4);
@@ -579,7 +566,7 @@ static qsf_hip_tensor* upload_locked(const void* host, int qt, int rows, int col
         free(fb);
     } else if (fmt < 0) {
         t->d_scales = base + off_scales;
-        he = mx_copy(t, p, t->payload_bytes);
+        he = mx_copy(t, p);
     } else {
         he = hipMemcpy(t->d_blocks, host_blocks, blocks_bytes, hipMemcpyHostToDevice);
     }
@@ -766,7 +753,7 @@ void qsf_hip_shutdown(void) {
         hipStreamSynchronize(g_dev.stream);
         if (g_dev.ws) hipFree(g_dev.ws);
         if (g_dev.att_ws) hipFree(g_dev.att_ws);
-        if (g_dev.h_up) hipHostFree(g_dev.h_up);
+        if (g_dev.d_up) hipFree(g_dev.d_up);
         if (g_dev.d_x) hipFree(g_dev.d_x);
         if (g_dev.slot_xq) hipFree(g_dev.slot_xq);
         if (g_dev.h_x) hipHostFree(g_dev.h_x);
@@ -1221,8 +1208,9 @@ struct qsf_hip_moe {
     size_t ws_bytes;
     void* d_many;            /* workspace of passes of more than 8 tokens, grown on demand */
     size_t many_bytes;
-    int chunks;              /* passes of 8 tokens only: a tensor is mx_wide, or has fewer
-                              * rows than the larger passes' loads take at a time (64) */
+    int chunks;              /* launches of 8 tokens only: a block scale is 2^126 or 2^127 (codes
+                              * 4 and 6 times it are outside bf16), or a tensor has fewer rows
+                              * than the larger passes' loads take at a time (64) */
     void* old[32];           /* outgrown ones: a captured graph may hold them */
     int n_old;
 };
@@ -1236,12 +1224,10 @@ qsf_hip_moe* qsf_hip_moe_create(int n_exp, int hidden, int eid,
         fail(E_INVALID, "qsf_hip_moe_create: bad arguments");
         return NULL;
     }
-    int chunks = hidden < 64 || eid < 64;
     for (int e = 0; e < n_exp; e++) {
         const qsf_hip_tensor* t[3] = {gate[e], up[e], down[e]};
         for (int i = 0; i < 3; i++) {
             int r = i < 2 ? eid : hidden, c = i < 2 ? hidden : eid;
-            if (t[i]) chunks |= t[i]->mx_wide;
             if (!t[i] || t[i]->fmt >= 0 || t[i]->rows != r || t[i]->cols != c) {
                 fail(E_INVALID, "qsf_hip_moe_create: expert %d tensor %d is not MXFP4 [%d][%d]",
                      e, i, r, c);
@@ -1285,9 +1271,17 @@ qsf_hip_moe* qsf_hip_moe_create(int n_exp, int hidden, int eid,
         rc = 1;
     free(host);
     m->n_exp = n_exp; m->hidden = hidden; m->eid = eid;
-    m->chunks = chunks;
     m->ws_bytes = qk_moe_ws_bytes(n_exp, 8, 8, hidden, eid);
     if (!rc && hipMalloc(&m->d_ws, m->ws_bytes) != hipSuccess) rc = 1;
+    m->chunks = hidden < 64 || eid < 64;
+    if (!rc && !m->chunks) {                                   /* or a scale of 2^126 or 2^127 */
+        int wide = 0;
+        if (qk_mx_wide(m->d_table, n_exp, hidden, eid, m->d_ws, g_dev.stream) ||
+            hipMemcpyAsync(&wide, m->d_ws, sizeof wide, hipMemcpyDeviceToHost, g_dev.stream) != hipSuccess ||
+            hipStreamSynchronize(g_dev.stream) != hipSuccess)
+            rc = 1;
+        m->chunks = wide != 0;
+    }
 
     if (rc) {
         if (m->d_ws) hipFree(m->d_ws);
