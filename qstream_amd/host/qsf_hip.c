@@ -1206,13 +1206,10 @@ struct qsf_hip_moe {
     void* d_alloc;           /* table + biases */
     void* d_ws;
     size_t ws_bytes;
-    void* d_many;            /* workspace of passes of more than 8 tokens, grown on demand */
-    size_t many_bytes;
-    int chunks;              /* launches of 8 tokens only: a block scale is 2^126 or 2^127 (codes
-                              * 4 and 6 times it are outside bf16), or a tensor has fewer rows
-                              * than the larger passes' loads take at a time (64) */
-    void* old[32];           /* outgrown ones: a captured graph may hold them */
-    int n_old;
+    void* d_many;            /* workspace of a pass of more than 16 tokens */
+    int chunks;              /* launches of 8 tokens only: no memory for d_many, a block scale is
+                              * 2^126 or 2^127 (codes 4 and 6 times it are outside bf16), or a
+                              * tensor has fewer rows than the passes' loads take at a time (64) */
 };
 
 qsf_hip_moe* qsf_hip_moe_create(int n_exp, int hidden, int eid,
@@ -1273,7 +1270,7 @@ qsf_hip_moe* qsf_hip_moe_create(int n_exp, int hidden, int eid,
     m->n_exp = n_exp; m->hidden = hidden; m->eid = eid;
     m->ws_bytes = qk_moe_ws_bytes(n_exp, 8, 8, hidden, eid);
     if (!rc && hipMalloc(&m->d_ws, m->ws_bytes) != hipSuccess) rc = 1;
-    m->chunks = hidden < 64 || eid < 64;
+    m->chunks = hidden < 64 || eid < 64 || hidden > 4096 || eid > 4096;
     if (!rc && !m->chunks) {                                   /* or a scale of 2^126 or 2^127 */
         int wide = 0;
         if (qk_mx_wide(m->d_table, n_exp, hidden, eid, m->d_ws, g_dev.stream) ||
@@ -1281,6 +1278,11 @@ qsf_hip_moe* qsf_hip_moe_create(int n_exp, int hidden, int eid,
             hipStreamSynchronize(g_dev.stream) != hipSuccess)
             rc = 1;
         m->chunks = wide != 0;
+    }
+    if (!rc && !m->chunks && hipMalloc(&m->d_many, qk_moe_many_ws_bytes(n_exp, hidden, eid)) != hipSuccess) {
+        (void)hipGetLastError();
+        m->d_many = NULL;
+        m->chunks = 1;
     }
 
     if (rc) {
@@ -1296,47 +1298,22 @@ qsf_hip_moe* qsf_hip_moe_create(int n_exp, int hidden, int eid,
 
 void qsf_hip_moe_free(qsf_hip_moe* m) {
     if (!m) return;
-    for (int i = 0; i < m->n_old; i++) hipFree(m->old[i]);
     if (m->d_many) hipFree(m->d_many);
     hipFree(m->d_ws);
     hipFree(m->d_alloc);
     free(m);
 }
 
-/* Workspace for a pass of ntok > 8 tokens: 1 when m->d_many holds it.  It
- * grows by half again as much as is asked for, so a few dozen growths reach
- * any size; an outgrown one stays until the object is freed.  Nothing is
- * allocated on a stream that is being captured. */
-static int many_ensure(qsf_hip_moe* m, int k, int ntok, hipStream_t s) {
-    const size_t need = qk_moe_many_ws_bytes(m->n_exp, k, ntok, m->hidden, m->eid);
-    pthread_mutex_lock(&g_lock);
-    if (m->many_bytes < need && m->n_old < 32) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        void* p = NULL;
-        if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
-            hipMalloc(&p, need + need / 2) == hipSuccess) {
-            if (m->d_many) m->old[m->n_old++] = m->d_many;
-            m->d_many = p;
-            m->many_bytes = need + need / 2;
-        } else {
-            (void)hipGetLastError();
-        }
-    }
-    const int ok = m->many_bytes >= need;
-    pthread_mutex_unlock(&g_lock);
-    return ok;
-}
-
 /* Up to MOE_MANY_MIN tokens run in the decode kernels, in chunks of 8; more
- * go through in passes of up to qk_moe_many_tokens(k) on the matrix cores,
- * or, where that workspace cannot be had (out of memory, or too small while
- * the stream is captured) or the tensors are not for them (m->chunks), in
- * chunks of 8 as well.  Where the line lies: 32 experts, top 4, 2880 x 2880: 9 tokens 101
+ * go through on the matrix cores, in as few passes of up to
+ * qk_moe_many_tokens(k) as hold them, all of about the same size; or, where
+ * the object has no workspace for them (m->chunks), in chunks of 8 as well.
+ * Where the line lies: 32 experts, top 4, 2880 x 2880: 9 tokens 101
  * us in chunks against 152 in a pass, 16 tokens 172 against 165 (8 experts,
  * top 2: 59 against 82 and 87 against 83); from 17 on a third chunk is due.
- * Chunks follow one another on `stream`, which orders their use of the
- * object's workspaces; a token's result does not depend on the
- * others in its chunk. */
+ * Chunks and passes follow one another on `stream`, which orders their use of
+ * the object's workspaces; a token's result does not depend on the others in
+ * its chunk or pass. */
 #define MOE_MANY_MIN 16
 
 static int g_moe_stages = 7;
@@ -1356,11 +1333,10 @@ int qsf_hip_moe_forward_dev(qsf_hip_moe* m, int k, int norm, int act, int ntok,
     const int stages = qsf_hip_moe_stages(-1);
     if (stages != 7 && ntok > 8)
         return fail(E_INVALID, "qsf_hip_moe_forward_dev: stages 0x%x need ntok <= 8 (one launch group)", stages);
-    const int most = qk_moe_many_tokens(k);
+    const int many = stages == 7 && ntok > MOE_MANY_MIN && !m->chunks, most = many ? qk_moe_many_tokens(k) : 8;
+    const int passes = ntok / most + (ntok % most != 0), each = many ? ntok / passes + (ntok % passes != 0) : 8;
     for (int t0 = 0, nt; t0 < ntok; t0 += nt) {
-        nt = ntok - t0 < most ? ntok - t0 : most;
-        const int many = stages == 7 && nt > MOE_MANY_MIN && !m->chunks && many_ensure(m, k, nt, pick_stream(stream));
-        if (!many && nt > 8) nt = 8;
+        nt = ntok - t0 < each ? ntok - t0 : each;
         const float *x = d_x + (size_t)t0 * m->hidden, *lg = d_logits + (size_t)t0 * m->n_exp;
         float* out = d_out + (size_t)t0 * m->hidden;
         if (many ? qk_moe_many_launch(m->d_table, m->n_exp, k, norm, act, m->hidden, m->eid, nt, x, lg, out,
