@@ -650,6 +650,8 @@ constexpr int FEW_P1 = 16 * 1024, FEW_T = 32 * 1024;       // a chunk's planes i
 constexpr int FEW_CHUNK = 36 * 1024;
 constexpr int FEW_XT = 2 * 1024;                           // rows of x: a wave's fragments being turned
 
+__device__ const uint8_t few_zero[16] __attribute__((aligned(16))) = {};
+
 template <int BS, int MT, int NT, bool PACKED>
 __global__ __launch_bounds__(FEW_WAVES * 64, 4) void prefill_few_kernel(FewArgs a) {
     constexpr int BB = 4 + BS / 2, P = BS / 64;            // block bytes, units a block
@@ -661,23 +663,29 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 4) void prefill_few_kernel(FewArgs 
     const size_t row_bytes = (size_t)a.nb * BB;
 
     // Chunk c into buffer `buf`: wave w loads rows 2 w and 2 w + 1 (rows past
-    // n and units past the row repeat the last one; neither is used)
+    // n and units past the row repeat the last one).  Units past the columns
+    // meet zeros of x; the piece with their scale and zero comes from few_zero (an
+    // infinite one times 0 is NaN).
+    const int nk = (a.k + 63) / 64;                        // units that hold columns
     auto load_chunk = [&](int c, uint8_t* buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int h = 0; h < 2 * NT; h++) {
             const int r = 2 * wave + (h & 1);              // row of tile h / 2
             const uint8_t* row = a.w + (size_t)min(n0 + 16 * (h >> 1) + r, a.n - 1) * row_bytes;
             uint8_t* tile = buf + (h >> 1) * FEW_CHUNK;
-            const int u = min(c * FEW_U + (lane ^ r), nu - 1);
-            const int ut = min(c * FEW_U + ((lane - 4 * r) & 63), nu - 1);
+            const int u0 = c * FEW_U + (lane ^ r), t0 = c * FEW_U + ((lane - 4 * r) & 63);
+            const int u = min(u0, nu - 1), ut = min(t0, nu - 1);
             // planes of a row: blocks of 64, {meta, codes 0-2}, {codes 3-6}, {code 7}
             // (dwords); larger blocks, {meta}, {codes 0-3}, {codes 4-7}
-            const uint8_t* p0 = row + (P == 1 ? 0 : 4 * a.nb) + 16 * (size_t)u;
-            const uint8_t* pt = P == 1 ? row + 32 * (size_t)a.nb + 4 * (size_t)ut : row + 4 * (size_t)(ut / P);
+            const uint8_t* p1 = row + (P == 1 ? 0 : 4 * a.nb) + 16 * (size_t)u;
+            const uint8_t* p0 = P == 1 && u0 >= nk ? few_zero : p1;
+            const uint8_t* pt = P == 1    ? row + 32 * (size_t)a.nb + 4 * (size_t)ut
+                                : t0 < nk ? row + 4 * (size_t)(ut / P)
+                                          : few_zero;
             typedef __attribute__((address_space(1))) void gvoid;
             typedef __attribute__((address_space(3))) void lvoid;
             __builtin_amdgcn_global_load_lds((gvoid*)p0, (lvoid*)(tile + r * 1024), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((gvoid*)(p0 + 16 * (size_t)nu), (lvoid*)(tile + FEW_P1 + r * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gvoid*)(p1 + 16 * (size_t)nu), (lvoid*)(tile + FEW_P1 + r * 1024), 16, 0, 0);
             __builtin_amdgcn_global_load_lds((gvoid*)pt, (lvoid*)(tile + FEW_T + r * 256), 4, 0, 0);
         }
     };
@@ -748,10 +756,8 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 4) void prefill_few_kernel(FewArgs 
             const uint8_t* buf = few_lds + i * NT * FEW_CHUNK;
 #pragma unroll
             for (int v = 0; v < 8; v++) {
+                if ((c0 + i) * FEW_U + 8 * v >= nu) break;
                 const int ul = 8 * v + wave;              // unit of the chunk
-                // (no unit of columns past k, where x is zero: an infinite scale
-                // or zero times that is NaN)
-                if (64 * ((c0 + i) * FEW_U + ul) >= a.k) break;
                 const uint32_t slot = (uint32_t)(n16 * 1024 + ((ul ^ n16) << 4));
                 const uint32_t ts = (uint32_t)(FEW_T + n16 * 256 + (((ul + 4 * n16) & 63) << 2));
                 uint32_t o0, o1, om;
