@@ -926,9 +926,13 @@ int few_gemm(const qsf_hip_tensor* t, const uint16_t* d_x, const void* d_ws, int
     // 4096, 64 tokens: 12.5 us in 128 workgroups of two tiles, 10.4 in 256 of
     // one; 128 tokens: 14.0 in 256 of two, 16.5 in 512 of one).
     const bool two = m > 32 && (long)((t->rows + 31) / 32) * ((m + 63) / 64) >= 256;
-    // chunks held at once: one workgroup a CU takes what LDS holds, more
-    // share it
-    const int fit = two ? 1 : tiles <= 256 && m <= 64 ? 4 : m <= 32 ? 2 : 1;
+    // chunks held at once: one workgroup a CU takes what LDS holds; where more
+    // share it, two with what half of it holds.  (Rows of x as they lie take the
+    // waves' turning space too, which leaves them one chunk: 2 x 8192 x 14336, blocks
+    // of 64, 25.6 us against 30.5 with two, one workgroup a CU; 16 x 4608 x 8192 13.1
+    // against 15.1.)
+    const int half = (80 * 1024 - (d_x ? FEW_WAVES * FEW_XT : 0)) / FEW_CHUNK;
+    const int fit = two ? 1 : tiles <= 256 && m <= 64 ? 4 : m <= 32 ? half : 1;
     FewArgs a = {t->d_blocks, d_x, static_cast<const u32x4*>(d_ws), d_y, m, t->rows, t->cols, t->nb,
                  4 * (st.sz + st.sc), 4 * st.sz, nch < fit ? nch : fit};
 #define QK_FEW(B, P)                                    \

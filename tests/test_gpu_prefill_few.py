@@ -22,11 +22,13 @@ def hip():
 # unit of K, fewer and more units than waves, a chunk's 64 units and one more,
 # all four chunks of a lone workgroup and a fifth, partial blocks of every
 # size, weight rows past a tile of 16 and of 32, enough workgroups for two
-# weight tiles each
+# weight tiles each, chunks held one (x as it lies) or two at a time by workgroups
+# that share a CU
 SHAPES = [(1, 15, 32, 64), (16, 17, 64, 64), (17, 33, 72, 64), (15, 16, 512, 64), (32, 31, 576, 64),
           (33, 40, 4096, 64), (64, 20, 4160, 64), (65, 48, 4168, 64), (3, 50, 16384, 64), (5, 18, 16456, 64),
           (40, 18, 20480, 64), (16, 100, 136, 128), (20, 70, 8264, 128), (64, 33, 264, 256), (9, 65, 16648, 256),
-          (100, 4100, 128, 64), (130, 2730, 200, 128), (128, 4096, 520, 256), (50, 8200, 4168, 64)]
+          (100, 4100, 128, 64), (130, 2730, 200, 128), (128, 4096, 520, 256), (50, 8200, 4168, 64),
+          (16, 4112, 8264, 128), (5, 5000, 12360, 64), (20, 4112, 12360, 64)]
 
 
 @pytest.mark.parametrize("m,n,k,bs", SHAPES)
