@@ -24,7 +24,7 @@
 // order (about 1e-6 rel-L2), not of bf16 weights.
 //
 // Tiling.  One 512-thread workgroup per 256 (m) x 112 (n) tile of Y (or 128
-// columns, qk_prefill_gemm); at config-4 shape (M 512, N 14336) 112 is exactly
+// columns, tile_cost); at config-4 shape (M 512, N 14336) 112 is exactly
 // one workgroup per CU.  K
 // advances in stages of 128 (4 MFMA k-steps): first the code stages, then
 // the zero-point stages (8 k positions per block, padded to an even stage
@@ -889,18 +889,33 @@ int gemm_check(const qsf_hip_tensor* t, int m) {
 }  // namespace
 
 namespace {
+// The tile kernel's time for m tokens, in sevenths of a round of 256 workgroups
+// of 112 columns; wide: with tiles of 128, where those take less (a round of 128
+// costs 8/7 of one of 112: 1999 x 4096 x 4096, 296 tiles of 112 in two rounds
+// 117 us with the pack, 256 of 128 in one 82 us).  Each output's arithmetic is the
+// same.
+long tile_cost(const qsf_hip_tensor* t, int m, bool& wide) {
+    auto rounds = [&](int bn) { return ((long)((t->rows + bn - 1) / bn) * ((m + BM - 1) / BM) + 255) / 256; };
+    const Stages st = stages_of(t->cols, t->bs);
+    const int bb = 4 + t->bs / 2;
+    wide = !t->frag && 8 * rounds(BN_MOST) < 7 * rounds(BN7) &&
+           (uint64_t)(t->rows + BN_MOST) * t->nb * bb + (uint64_t)16 * st.sz * bb < (1ull << 32);
+    return wide ? 8 * rounds(BN_MOST) : 7 * rounds(BN7);
+}
+
 // Whether the few-token kernel takes m tokens of a tensor: where its time, in
 // proportion to its workgroups (0.157 us a unit of K and 256 of them), is below
-// the tile kernel's, in proportion to its rounds of 256 workgroups (0.84 us a
-// unit and round).  GEMM alone, few against tile, us: 4096 x 4096, 16 tokens 5.0
-// / 54.6, 256 22.9 / 58.9, 512 43.2 / 58; 4096 x 11008, 64 tokens 23.3 / 143.7, 512
-// 117 / 146; 14336 x 4096, 64 tokens 24.5 / 58.4, 128 44 / 59, 256 80 / 58.
-// (Fragment-order tensors keep to the tile kernel.)
+// the tile kernel's (0.84 us a unit and round of 112).  GEMM alone, few against
+// tile, us: 4096 x 4096, 16 tokens 5.0 / 54.6, 256 22.9 / 58.9, 512 43.2 / 58;
+// 4096 x 11008, 64 tokens 23.3 / 143.7, 512 117 / 146; 14336 x 4096, 64 tokens
+// 24.5 / 58.4, 128 44 / 59, 256 80 / 58; with the pack, against one round of 128:
+// 16384 x 4096, 257 tokens 97.6 / 83.7, 320 105 / 85; 32768 x 2048, 128 tokens 54.4
+// / 48.6.  (Fragment-order tensors keep to the tile kernel.)
 bool few_takes(const qsf_hip_tensor* t, int m) {
     if (t->frag) return false;
     const long wgs = (long)((t->rows + 31) / 32) * ((m + 63) / 64);
-    const long rounds = ((long)((t->rows + BN7 - 1) / BN7) * ((m + BM - 1) / BM) + 255) / 256;
-    return wgs < 1360 * rounds;
+    bool wide;
+    return 7 * wgs < 1360 * tile_cost(t, m, wide);
 }
 
 template <int BS, int MT, int NT, bool PACKED>
@@ -966,14 +981,9 @@ extern "C" int qk_prefill_gemm(const qsf_hip_tensor* t, const void* d_ws, int m,
     const uint64_t row_bytes = (uint64_t)t->nb * bb;
     const bool ragged = t->cols % (2 * SK) != 0;
     const uint64_t w_bytes = t->frag ? (uint64_t)qk_frag_bytes(t->rows, t->nb, bb) : (uint64_t)t->rows * row_bytes;
-    // Columns of a tile: 112, or 128 where that takes fewer rounds of 256
-    // workgroups (a round of 128 costs 8/7 of one of 112: 1999 x 4096 x 4096, 296
-    // tiles of 112 in two rounds 121 us with the pack, 256 of 128 in one 89 us).  Each
-    // output's arithmetic is the same.
-    auto rounds = [&](int bn) { return ((long)((t->rows + bn - 1) / bn) * tiles_m + 255) / 256; };
-    const bool wide = !t->frag && 8 * rounds(128) < 7 * rounds(112) &&
-                      (uint64_t)(t->rows + BN_MOST) * row_bytes + (uint64_t)16 * st.sz * bb < (1ull << 32);
-    const int bn = wide ? 128 : 112, zp_max = wide ? Tile<8>::ZP_MAX : Tile<7>::ZP_MAX;
+    bool wide;
+    (void)tile_cost(t, m, wide);
+    const int bn = wide ? BN_MOST : BN7, zp_max = wide ? Tile<8>::ZP_MAX : Tile<7>::ZP_MAX;
     const int tiles_n = (t->rows + bn - 1) / bn;
     PrefillArgs a = {t->d_blocks, static_cast<const u32x4*>(d_ws), d_y, m, t->rows, t->cols, t->nb,
                      tiles_n, st.sz, st.sz + st.sc, 16 * st.sz <= zp_max ? 16 * st.sz : 0,

@@ -115,3 +115,19 @@ def test_wide_tiles(hip, oracle, m, n, k, bs):
     err = rel_l2(got[np.ix_(toks, rows)], ref)
     print(f"wide tiles {m}x{n}x{k} bs{bs}: rel_l2 {err:.3e}")
     assert err <= REL_L2
+
+
+# (rows, tokens, tile): one round of tiles of 128 columns against two of 112 (the
+# tile kernel from 257 to 320 tokens), 2 M tiles of them, and sizes beside them
+# that the few-token kernel keeps (its workgroups cost less than a round)
+@pytest.mark.parametrize("n,m,tile", [(16384, 257, True), (16384, 320, True), (14337, 257, True), (32768, 128, True),
+                                      (14336, 128, False), (4096, 257, False), (8192, 320, False)])
+def test_few_or_tile(hip, n, m, tile):
+    """Which kernel took a call, by its bits: those of the first m tokens of a
+    call too large for the few-token kernel, or not."""
+    k, bs, most = 328, 64, 1030
+    payload, xb = case(n + m, most, n, k, bs)
+    got = run(hip, payload, xb[:m], m, n, k, bs)
+    ref = run(hip, payload, xb, most, n, k, bs)[:m]
+    assert rel_l2(got, ref) <= REL_L2
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)) == tile
