@@ -238,8 +238,9 @@ typedef struct qsf_hip_moe qsf_hip_moe;         /* opaque device expert table */
  * expert (the MOE_*_BIAS tensors, src/engine.c:1039-1046); the outer array or
  * any entry may be NULL.  Device memory beside the tensors: 1.5 MB at
  * 2880 x 2880, and the workspace of the passes of more than 16 tokens, 96 bytes
- * times (hidden + expert_dim, each rounded up to 256) times
- * (128 + n_experts): 94 MB at 32 experts of 2880 x 2880. */
+ * times (hidden + expert_dim, each rounded up to 256) times (64 for up to 16
+ * experts, 256 from 64 on, else 4 * n_experts; plus n_experts): 94 MB at 32
+ * experts of 2880 x 2880. */
 qsf_hip_moe* qsf_hip_moe_create(int n_experts, int hidden, int expert_dim,
                                 const qsf_hip_tensor* const* gate,
                                 const qsf_hip_tensor* const* up,
@@ -254,12 +255,13 @@ void qsf_hip_moe_free(qsf_hip_moe* m);
  * ReLU) times up, down + bias, weighted sum in rank order.  d_x [ntok][hidden],
  * d_logits [ntok][n_experts], d_out [ntok][hidden]; asynchronous, in order on
  * `stream`, and nothing is allocated.  Up to 16 tokens run in launches of 8;
- * more on the matrix cores, in passes of up to 2048 / top_k tokens (in
- * launches of 8 as well where hidden or expert_dim is below 64, a block scale
- * of any expert is 2^126 or 2^127, or _create had no memory for the passes'
- * workspace).  A token's result does not depend on the other tokens of the
- * call; launches and passes add in different orders, so its last bits do
- * depend on whether the call has more than 16 tokens.  The workspaces belong
+ * more on the matrix cores, in passes of up to P / top_k tokens, P = 64 *
+ * n_experts but at least 1024 and at most 4096 (in launches of 8 as well where
+ * hidden or expert_dim is below 64, a block scale of any expert is 2^126 or
+ * 2^127, or _create had no memory for the passes' workspace).  A token's
+ * result does not depend on the other tokens of the call; launches and passes
+ * add in different orders, so its last bits do depend on whether the call has
+ * more than 16 tokens.  The workspaces belong
  * to the object: calls with one object must not overlap. */
 int qsf_hip_moe_forward_dev(qsf_hip_moe* m, int top_k, int norm_topk, int activation,
                             int ntok, const float* d_x, const float* d_logits,

@@ -212,9 +212,9 @@ int qk_mx_split(const uint8_t* codes, const uint8_t* scales, uint8_t* d_blocks, 
 int qk_mx_wide(const qk_mx_expert* d_experts, int n_exp, int hidden, int eid, int* d_flag, hipStream_t s);
 
 /* The FFN for many tokens in one pass on the matrix cores: up to
- * qk_moe_many_tokens(k) tokens, with a workspace of qk_moe_many_ws_bytes (for
+ * qk_moe_many_tokens tokens, with a workspace of qk_moe_many_ws_bytes (for
  * any k). */
-int qk_moe_many_tokens(int k);
+int qk_moe_many_tokens(int n_exp, int k);
 size_t qk_moe_many_ws_bytes(int n_exp, int hidden, int eid);
 int qk_moe_many_launch(const qk_mx_expert* d_experts, int n_exp, int k, int norm, int act,
                        int hidden, int eid, int ntok, const float* d_x, const float* d_logits,

@@ -1306,7 +1306,7 @@ void qsf_hip_moe_free(qsf_hip_moe* m) {
 
 /* Up to MOE_MANY_MIN tokens run in the decode kernels, in chunks of 8; more
  * go through on the matrix cores, in as few passes of up to
- * qk_moe_many_tokens(k) as hold them, all of about the same size; or, where
+ * qk_moe_many_tokens as hold them, all of about the same size; or, where
  * the object has no workspace for them (m->chunks), in chunks of 8 as well.
  * Where the line lies: 32 experts, top 4, 2880 x 2880: 9 tokens 101
  * us in chunks against 152 in a pass, 16 tokens 172 against 165 (8 experts,
@@ -1333,7 +1333,7 @@ int qsf_hip_moe_forward_dev(qsf_hip_moe* m, int k, int norm, int act, int ntok,
     const int stages = qsf_hip_moe_stages(-1);
     if (stages != 7 && ntok > 8)
         return fail(E_INVALID, "qsf_hip_moe_forward_dev: stages 0x%x need ntok <= 8 (one launch group)", stages);
-    const int many = stages == 7 && ntok > MOE_MANY_MIN && !m->chunks, most = many ? qk_moe_many_tokens(k) : 8;
+    const int many = stages == 7 && ntok > MOE_MANY_MIN && !m->chunks, most = many ? qk_moe_many_tokens(m->n_exp, k) : 8;
     const int passes = ntok / most + (ntok % most != 0), each = many ? ntok / passes + (ntok % passes != 0) : 8;
     for (int t0 = 0, nt; t0 < ntok; t0 += nt) {
         nt = ntok - t0 < each ? ntok - t0 : each;
