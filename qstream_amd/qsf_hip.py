@@ -284,12 +284,11 @@ class KernelTable:
     def _slot(self, fn):
         def call(w, x, out, rows, cols, bs):
             wa = np.frombuffer(w, np.uint8) if isinstance(w, (bytes, bytearray)) else w
-            pw = wa.ctypes.data
-            self._keep.setdefault(pw, wa)   # the library keys uploaded payloads by address
+            self._keep.setdefault(wa.ctypes.data, wa)   # the library keys uploaded payloads by address
             if not (out.dtype == np.float32 and out.flags.c_contiguous):
                 raise TypeError("output must be a contiguous float32 array")
             xa = np.ascontiguousarray(x, np.float32)
-            fn(pw, xa.ctypes.data, out.ctypes.data, rows, cols, bs)
+            fn(wa.ctypes.data, xa.ctypes.data, out.ctypes.data, rows, cols, bs)
         return call
 
 
