@@ -279,16 +279,17 @@ class KernelTable:
         self._L = load()
         for s in MATVEC_SLOTS + ("matvec_mxfp4",):
             setattr(self, s, self._slot(getattr(self._L, f"qsf_{s}_hip")))
-        self._keep = []
+        self._keep = {}
 
     def _slot(self, fn):
         def call(w, x, out, rows, cols, bs):
             wa = np.frombuffer(w, np.uint8) if isinstance(w, (bytes, bytearray)) else w
-            self._keep.append(wa)   # the library keys uploaded payloads by address
+            pw = wa.ctypes.data
+            self._keep.setdefault(pw, wa)   # the library keys uploaded payloads by address
             if not (out.dtype == np.float32 and out.flags.c_contiguous):
                 raise TypeError("output must be a contiguous float32 array")
             xa = np.ascontiguousarray(x, np.float32)
-            fn(wa.ctypes.data, xa.ctypes.data, out.ctypes.data, rows, cols, bs)
+            fn(pw, xa.ctypes.data, out.ctypes.data, rows, cols, bs)
         return call
 
 

@@ -100,6 +100,21 @@ def _load_fresh(mod, path):
         mod._lib = saved
 
 
+def test_kernel_table_keeps_a_payload_once():
+    """The binding holds each payload's memory (uploads are keyed by its address)
+    once, not once a call."""
+    import numpy as np
+    from qstream_amd import qsf_hip
+    kt = qsf_hip.KernelTable()
+    seen = []
+    call = kt._slot(lambda w, x, y, *shape: seen.append(w))
+    payloads = [bytes(36), bytearray(36), np.zeros(36, np.uint8)]
+    for _ in range(50):
+        for w in payloads:
+            call(w, np.zeros(64, np.float32), np.empty(1, np.float32), 1, 64, 64)
+    assert len(kt._keep) == len(set(seen)) == 3
+
+
 DROPIN = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle", "_ref",
                       "dropin_table")
 
