@@ -286,8 +286,10 @@ int qsf_hip_moe_stages(int mask);
  * on MFMA with fp32 accumulation, the scale is applied in fp32 every 64
  * codes, and the zero-point term runs on exact bf16 splits of z and of the
  * block sums; nothing is rounded below fp32 (about 1e-6 rel-L2 against the
- * scalar matvec on float(x)).  d_x is bf16 [m][cols] (16-byte aligned,
- * cols >= 32, cols % 8 == 0); asynchronous on `stream`.  Uses the library
+ * scalar matvec on float(x)).  A token's result does not depend on the other
+ * tokens of the call, but its last bits depend on their number: calls of few
+ * tokens run in a kernel of their own, which adds in another order.  d_x is bf16
+ * [m][cols] (16-byte aligned, cols >= 32, cols % 8 == 0); asynchronous on `stream`.  Uses the library
  * workspace (x repacked into fragment order with the block-sum splits,
  * about 2*m*cols bytes plus 16 per block and token): calls must not overlap
  * with other workspace users on other streams.  The workspace grows as
@@ -304,7 +306,8 @@ int qsf_hip_prefill_4bit_dev(const qsf_hip_tensor* t, const uint16_t* d_x_bf16, 
  * workspace, and nothing is allocated or freed.  A call that needs more
  * scratch than that (about 2 * m * (cols + 8 * cols / block_size) bytes,
  * m rounded up to 16 and both column counts to 256; config 4's 512 x 4096
- * at block 64 needs 4.7 MB) fails with QSF_ERR_INVALID_INPUT.  Every call on one GPU shares that GPU's
+ * at block 64 needs 4.7 MB) fails with QSF_ERR_INVALID_INPUT (split the tokens
+ * over calls, whose last bits may then differ).  Every call on one GPU shares that GPU's
  * array: calls that overlap on one GPU (different streams, or graphs
  * replayed concurrently) race on it. */
 #define QSF_HIP_PREFILL_SCRATCH_BYTES (16 << 20)

@@ -361,9 +361,9 @@ __global__ __launch_bounds__(64) void rope_kv_kernel(float* q, float* k, const f
 //    position groups by halving (each step exchanges half of the values with
 //    the lanes 32, 16, 8 or 4 away and adds), then over the waves in LDS.
 // Measured with the merge below (32 heads on 8 KV heads of 128, 12345 positions, graph
-// replay, 26 MB of cache): 68.2 -> 19.3 us a step against one workgroup a
+// replay, 26 MB of cache): 68.2 -> 19.4 us a step against one workgroup a
 // (head, chunk), an LDS pass over 32 partial rows an output and the serial
-// merge; a 7B layer step (1024 positions, MHA, G = 1) 49.3 -> 48.4 us.
+// merge; a 7B layer step (1024 positions, MHA, G = 1) 49.3 -> 48.2 us.
 // The arithmetic of a head does not depend on G, nor on FUSED: the cache
 // rows, scales and chunk records of the fused launch equal those of
 // rope_kv_kernel followed by the plain one bit for bit.

@@ -892,7 +892,7 @@ namespace {
 // The tile kernel's time for m tokens, in sevenths of a round of 256 workgroups
 // of 112 columns; wide: with tiles of 128, where those take less (a round of 128
 // costs 8/7 of one of 112: 1999 x 4096 x 4096, 296 tiles of 112 in two rounds
-// 117 us with the pack, 256 of 128 in one 82 us).  Each output's arithmetic is the
+// 117 us with the pack, 256 of 128 in one 81 us).  Each output's arithmetic is the
 // same.
 long tile_cost(const qsf_hip_tensor* t, int m, bool& wide) {
     auto rounds = [&](int bn) { return ((long)((t->rows + bn - 1) / bn) * ((m + BM - 1) / BM) + 255) / 256; };

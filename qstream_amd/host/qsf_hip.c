@@ -407,8 +407,9 @@ static void plane_permute(uint8_t* dst, const uint8_t* src, int rows, int nb, in
 /* An MXFP4 payload to the tensor's planes (qk_mx_at).  Where that is the
  * on-disk order (a multiple of 8 blocks a row, or fewer than 8) as it is;
  * else by the piece through a device buffer, from which a kernel moves each
- * row's whole groups of 8 blocks and its remainder to their planes.  Done when it
- * returns: a caller may use the tensor on any stream. */
+ * row's whole groups of 8 blocks and its remainder to their planes (96 tensors of
+ * 2880 x 2880, 90 blocks a row: 26 ms, 24.5 as they are).  Done when it returns: a
+ * caller may use the tensor on any stream. */
 #define UP_PIECE ((size_t)8 << 20)
 static hipError_t mx_copy(qsf_hip_tensor* t, const uint8_t* payload) {
     const size_t rows = (size_t)t->rows, nb = (size_t)t->nb;
@@ -1308,9 +1309,10 @@ void qsf_hip_moe_free(qsf_hip_moe* m) {
  * go through on the matrix cores, in as few passes of up to
  * qk_moe_many_tokens as hold them, all of about the same size; or, where
  * the object has no workspace for them (m->chunks), in chunks of 8 as well.
- * Where the line lies: 32 experts, top 4, 2880 x 2880: 9 tokens 101
- * us in chunks against 152 in a pass, 16 tokens 172 against 165 (8 experts,
- * top 2: 59 against 82 and 87 against 83); from 17 on a third chunk is due.
+ * Where the line lies: 32 experts, top 4, 2880 x 2880: 9 tokens 106 us in
+ * chunks against 140 in a pass, 12 tokens 134 against 147, 16 tokens 165 against
+ * 155 (8 experts, top 2: 60 / 75, 75 / 76, 89 / 76); from 17 on a third chunk is
+ * due.
  * Chunks and passes follow one another on `stream`, which orders their use of
  * the object's workspaces; a token's result does not depend on the others in
  * its chunk or pass. */
